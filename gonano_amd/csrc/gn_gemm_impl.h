@@ -31,11 +31,6 @@ struct GemmParams {
   // batched products (grid y): product y reads A + y*bsa, B + y*bsb and
   // writes C + y*bsc, its split partials [splits][M][N] at part + y*splits*M*N
   int64_t bsa, bsb, bsc;
-  // wide engine: bits of the largest |value| of every A row m and B row n,
-  // over achunks (bchunks) ranges of k: [chunks][rows]
-  const uint32_t* amax;
-  const uint32_t* bmax;
-  int achunks, bchunks;
 };
 
 // Workgroup -> (tile row, tile column, split).  Workgroups are dealt to the

@@ -140,7 +140,7 @@ struct GemmDesc {
 
 // Which kernel ran a product: gemm_kernel (tiles up to 128 x 128, fused
 // epilogues, grouped and deferred products), the wide-tile engine (the large
-// products, on the fp16 matrix cores; gn_gemm_wide.hip), the slim-tile
+// products, on the bf16 matrix cores; gn_gemm_wide.hip), the slim-tile
 // engine (32-row tiles for the decode projections) or the skinny engine
 // (at most 32 rows; gn_gemm_skinny.hip).
 enum GemmEngine {

@@ -242,11 +242,10 @@ def test_attention(be, orc, qlen, klen, dim, offset, window, seg):
 
 @pytest.mark.parametrize("m,n,k", [(2000, 6000, 512), (4096, 3072, 768), (256, 12288, 1024)])
 def test_matmul_wide_engine(be, m, n, k):
-    """Products large enough for the 256 x 256-tile engine (at least 192
-    workgroups): MatMulTransposed (x.W^T, both operands K-contiguous) and
-    MatMul (B contiguous in N), against numpy in float64.  2000 x 6000
-    leaves a partial last tile in both dimensions (loaded shifted back to
-    end at M and N, the overlap not stored twice)."""
+    """Products large enough for the wide-tile engine: MatMulTransposed
+    (x.W^T, both operands K-contiguous) and MatMul (B contiguous in N), against
+    numpy in float64.  2000 x 6000 leaves a partial last tile in both
+    dimensions."""
     rng = np.random.default_rng(m + n + k)
     a = rng.standard_normal((m, k)).astype(f32)
     b = rng.standard_normal((k, n)).astype(f32)
@@ -283,49 +282,80 @@ def test_matmul_slim_engine(be, monkeypatch, m, n, k, mode):
     assert_close(got, want, 1e-4, 1e-4, "MatMulTransposed")
 
 
-@pytest.mark.parametrize("tile", ["128", "256"])
+def _split_bound(a, w):
+    """Largest error per output of the wide-tile engine's three-term bf16
+    products: the parts hold every bit; the dropped terms are at most 2^-24 of
+    each |a||b|; each of the 6K/16 accumulating instructions rounds its 16
+    products and the sum, at most 17 units of 2^-24 of sum |a||b|, which covers
+    the K + 2 roundings of the plain fp32 sums; and float32's last subnormal."""
+    k = a.shape[1]
+    return (2.0 ** -24 + 17 * 2.0 ** -24 * (6 * k / 16 + 3)) * \
+        (np.abs(a.astype(np.float64)) @ np.abs(w.astype(np.float64)).T) + 2.0 ** -149
+
+
+def _check_split(be, a, w, bound, what):
+    m, k, n = *a.shape, w.shape[0]
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = a.astype(np.float64) @ w.astype(np.float64).T
+        want32 = want.astype(f32)
+    fin = np.isfinite(want32)
+    for name in ("MatMulTransposed", "MatMul"):
+        got = np.full((m, n), -7.0, f32)
+        if name == "MatMul":
+            be.MatMul(got, a, np.ascontiguousarray(w.T), m, n, k)
+        else:
+            be.MatMulTransposed(got, a, w, m, n, k)
+        assert np.all(np.abs(got.astype(np.float64) - want)[fin] <= bound[fin]), (what, name)
+        assert np.array_equal(got[~fin], want32[~fin], equal_nan=True), (what, name)
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 4, 8), (127, 132, 40), (129, 260, 776), (256, 256, 32),
                                    (300, 516, 1000)])
-def test_matmul_split_products(be, monkeypatch, m, n, k, tile):
-    """The wide-tile engine's two-term fp16 split at the edges of its tiles and
-    K steps, on rows and columns of magnitudes 2^-60 .. 2^60 (a power-of-two
-    scale per row leaves no trace), a zero row, and a row and a column that
-    hold an infinity or a NaN (plain fp32 sums there; the others untouched).
-    Bound per output: the split loses at most 2^-22 of each |a||b| and every
-    one of the 3K/16 accumulating instructions rounds its 16 products and the
-    sum, at most 17 units of 2^-24 of sum |a||b|, so (2^-22 + 17 * 2^-24 *
-    (3K/16 + 3)) * |A||B|^T."""
+def test_matmul_split_products(be, monkeypatch, m, n, k):
+    """The wide-tile engine at the edges of its tiles and K steps, on rows and
+    columns of magnitudes 2^-60 .. 2^60, a zero row, and a row and a column
+    that hold an infinity or a NaN (plain fp32 sums there; the others
+    untouched)."""
     monkeypatch.setenv("GN_GEMM_WIDE_MIN", "1")
-    monkeypatch.setenv("GN_GEMM_WIDE_TILE", tile)
     rng = np.random.default_rng(m + n + k)
     a = rng.standard_normal((m, k)).astype(f32)
     w = rng.standard_normal((n, k)).astype(f32)
     a *= np.exp2(rng.integers(-60, 61, (m, 1))).astype(f32)
     w *= np.exp2(rng.integers(-60, 61, (n, 1))).astype(f32)
-    a[m // 2] = 0
-    bound = (2.0 ** -22 + 17 * 2.0 ** -24 * (3 * k / 16 + 3)) * \
-        (np.abs(a.astype(np.float64)) @ np.abs(w.astype(np.float64)).T)
-
-    def check(what):
-        want = a.astype(np.float64) @ w.astype(np.float64).T
-        fin = np.isfinite(want)
-        for name, got in (("MatMulTransposed", np.zeros((m, n), f32)),
-                          ("MatMul", np.zeros((m, n), f32))):
-            if name == "MatMul":
-                be.MatMul(got, a, np.ascontiguousarray(w.T), m, n, k)
-            else:
-                be.MatMulTransposed(got, a, w, m, n, k)
-            assert np.all(np.abs(got - want)[fin] <= bound[fin]), (what, name)
-            assert np.array_equal(np.isnan(got), np.isnan(want)), (what, name)
-            inf = np.isinf(want)
-            assert np.array_equal(got[inf], want[inf].astype(f32)), (what, name)
-
-    check("finite")
     if m > 1:
-        with np.errstate(invalid="ignore"):
-            a[0, 0], w[1, k - 1] = np.inf, np.nan
-            bound[0, :] = bound[:, 1] = 0  # those outputs are infinite or NaN
-            check("non-finite")
+        a[m // 2] = 0
+    bound = _split_bound(a, w)
+    _check_split(be, a, w, bound, "finite")
+    a[0, 0], w[1, k - 1] = np.inf, np.nan
+    _check_split(be, a, w, bound, "non-finite")
+
+
+@pytest.mark.parametrize("m,n,k", [(130, 260, 72), (257, 132, 800)])
+def test_matmul_split_range(be, monkeypatch, m, n, k):
+    """Operands whose rows hold magnitudes far apart: large entries that meet
+    zeros of the other operand (2^30, 2^60, and a lowest-value sentinel), every
+    magnitude from float32's subnormals up, and values and sums beyond the
+    bf16 parts' range, which take plain fp32 sums.  The bound is per output
+    and relative to its own terms, so nothing large elsewhere excuses an error."""
+    monkeypatch.setenv("GN_GEMM_WIDE_MIN", "1")
+    rng = np.random.default_rng(m + n + k)
+    base_a = rng.standard_normal((m, k)).astype(f32)
+    base_w = rng.standard_normal((n, k)).astype(f32)
+    for big in (2.0 ** 30, 2.0 ** 60, -1e30):
+        a, w = base_a.copy(), base_w.copy()
+        a[:, 3], w[:, 3] = big, 0
+        w[:, k - 1], a[:, k - 1] = big, 0
+        _check_split(be, a, w, _split_bound(a, w), f"large entry {big:g} against zeros")
+    a = np.ldexp(base_a, rng.integers(-148, 20, (m, k))).astype(f32)
+    w = np.ldexp(base_w, rng.integers(-30, 60, (n, k))).astype(f32)
+    _check_split(be, a, w, _split_bound(a, w), "all magnitudes")
+    # one tile's rows above 2^104, sums above 2^81, and an overflowing one
+    a, w = base_a.copy(), np.abs(base_w) + f32(0.5)
+    a[1] = np.ldexp(np.abs(a[1]) + f32(1), 110)
+    w[0] = np.ldexp(w[0], -60)
+    w[2] = np.ldexp(w[2], 85)
+    w[n - 1] = np.ldexp(w[n - 1], 30)
+    _check_split(be, a, w, _split_bound(a, w), "beyond the split's range")
 
 
 @pytest.mark.parametrize("m", [1, 15, 17, 32])

@@ -467,6 +467,44 @@ def test_latent_width_pg_step_wide_grouped_k(orc, latw, monkeypatch, parts):
     assert n_on == n_off and on - off == 3 * cfg.n_layer, (on, off, n_on)
 
 
+def test_latent_width_expert_gradients_keep_their_own_range(latw, monkeypatch):
+    """Expert weight gradients are independent sums over each expert's rows: a
+    sequence whose gradients are 2^50 times the other's must not cost the
+    experts that it does not reach any bits.  Those are the experts whose
+    gradient is zero when the other sequence carries no loss; theirs equal
+    the gradients without the large sequence."""
+    from gonano_amd.session import Session
+    cfg, w = latw
+    cfg = dataclasses.replace(cfg, balance_weight=0.0)
+    monkeypatch.setenv("GN_GEMM_WIDE_MIN", "1")
+    rng = np.random.default_rng(5)
+    T = 200
+    inputs = rng.integers(0, cfg.vocab_size, (2, T)).astype(np.int32)
+    targets = rng.integers(0, cfg.vocab_size, (2, T)).astype(np.int32)
+    targets[0, 2:] = -1  # the large sequence's gradient reaches two tokens
+    with Session(cfg) as s:
+        s.set_params(w)
+
+        def grads(a0, a1):
+            s.zero_grad()
+            s.policy_gradient_step(inputs, targets, np.array([a0, a1], np.float32), 1.0)
+            return s.grads()
+
+        both, small, large = grads(2.0 ** 50, 1.0), grads(0.0, 1.0), grads(2.0 ** 50, 0.0)
+    checked = 0
+    for name, rows, cols, off in cfg.param_table():
+        if ".experts." not in name:
+            continue
+        E = cfg.n_experts
+        pick = lambda g: g[off:off + rows * cols].reshape(E, -1)
+        for e in range(E):
+            if pick(large)[e].any() or not pick(small)[e].any():
+                continue
+            checked += 1
+            assert rel_err(pick(both)[e], pick(small)[e]) <= 1e-5, (name, e)
+    assert checked >= 3, checked
+
+
 # ---- flash d12 width (the benchmark's flash d12 workload at 6 layers, V 4096) ---
 @pytest.fixture(scope="module")
 def flashw():
