@@ -11,8 +11,8 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -91,12 +91,15 @@ class HostCopy {
       if (e != hipSuccess) return;  // the others take its share
       for (size_t j; !failed() && (j = taken.fetch_add(1)) < n;) drain(j);
     };
+    // Nothing between the first thread and the joins may throw: a thread (or
+    // its memory) that cannot be had means fewer helpers, the caller takes
+    // the rest.
+    const size_t helpers = std::min<size_t>(THREADS, n) - 1;
     std::vector<std::thread> threads;
+    threads.reserve(helpers);
     try {
-      const size_t helpers = std::min<size_t>(THREADS, n) - 1;
       for (size_t l = 0; l < helpers; l++) threads.emplace_back(helper);
-    } catch (const std::system_error&) {
-      // fewer helpers: the caller takes the rest
+    } catch (const std::exception&) {
     }
     for (size_t i = 0; i < n && !failed();) {
       if (freed[i % slots].load(std::memory_order_acquire) == i / slots) {
