@@ -225,11 +225,10 @@ def test_d12_width_pg_step_chunked(orc, d12w, monkeypatch):
 
 
 def test_d12_width_pg_step_wide_engine(orc, d12w, monkeypatch):
-    """The policy-gradient step with every product the 256 x 256-tile engine
-    can take routed there at any grid size (GN_GEMM_WIDE_MIN=1; the
-    benchmark's 130,816-token products take it by size): 4 x 512 tokens
-    make every M, N >= 256 and every K a multiple of 64, so the instances
-    run are the forward products (plain qkv, residual-add wo, ReLU^2 fc
+    """The policy-gradient step with every product the wide-tile engine can
+    take routed there at any size (GN_GEMM_WIDE_MIN=1; the benchmark's
+    130,816-token products take it by size): the instances run are the
+    forward products (plain qkv, residual-add wo, ReLU^2 fc
     with the saved pre-activation, the proj product as split-K partials
     with the residual add in the reduction), the input gradients (plain,
     ReLU^2 backward, split-K partials), the weight gradients (split-K
@@ -261,10 +260,9 @@ def test_d12_width_pg_step_tile_engine(orc, d12w, monkeypatch):
 
 def test_d12_width_pg_step_wide_engine_ragged_k(orc, d12w, monkeypatch):
     """As above with 4 x 500 tokens: the weight gradients' K (2000 tokens) is
-    not a multiple of 64, so the engine runs K in [0, 1984) as its splits
-    and the last 16 tokens as one more split on gemm_kernel, summed with the
-    others by the reduction (the flash and d20 workloads' token counts,
-    16 x 8703 and B x 1535, take this path)."""
+    not a multiple of the engine's 32-deep stages, so the last K range ends
+    inside one and reads zeros past its end (the flash and d20 workloads'
+    token counts, 16 x 8703 and B x 1535, do the same)."""
     cfg, w = d12w
     monkeypatch.setenv("GN_GEMM_WIDE_MIN", "1")
     t = _pg_check(orc, cfg, w, B=4, T=500, prompt_len=372, chunk=256, monkeypatch=monkeypatch,
@@ -321,6 +319,33 @@ def test_d12_width_few_rows_rollout(orc, d12w, groups, samples):
     _rollout_check(orc, cfg, w, groups, samples, 140, 8, 1.0, [0])
 
 
+@pytest.mark.parametrize("C", [256, 512, 768, 1024, 1280, 1536])
+def test_few_row_norm_widths(C, monkeypatch):
+    """The MLP norm inside the few-row input projection at every width it takes
+    (one 16-row block up to 1536, two up to 768) against the separate norm
+    (GN_FUSE_NORM=0), and the few-row engine against the others
+    (GN_GEMM_SKINNY=0): the same sampled tokens."""
+    from gonano_amd.session import Session
+    cfg = dataclasses.replace(d12_width(), n_embd=C, n_head=C // 128,
+                              n_kv_head=2 if C > 1024 else C // 256)
+    w = G.init_weights(cfg, seed=C, perturb=0.05)
+    prompts = np.random.default_rng(C).integers(0, cfg.vocab_size, (1, 40)).astype(np.int32)
+    seeds = np.array([77], np.uint64)
+    for samples in (1, 16, 17):
+        rows = []
+        for env in ({}, {"GN_FUSE_NORM": "0"}, {"GN_GEMM_SKINNY": "0", "GN_FUSE_NORM": "0"}):
+            for k, v in env.items():
+                monkeypatch.setenv(k, v)
+            with Session(cfg) as s:
+                s.set_params(w)
+                rows.append(s.generate_batch(prompts, samples, 12, 1.0, 50, seeds))
+            for k in env:
+                monkeypatch.delenv(k)
+        for other in rows[1:]:
+            assert len(other) == samples
+            assert all(np.array_equal(a, b) for a, b in zip(rows[0], other)), (C, samples)
+
+
 # ---- d12 width at the benchmark's vocabulary (V = 65536) --------------------
 @pytest.fixture(scope="module")
 def d12v():
@@ -340,7 +365,7 @@ def test_d12_vocab_pg_step_chunked(orc, d12v, monkeypatch):
 
 def test_d12_vocab_pg_step_wide_engine(orc, d12v, monkeypatch):
     """The same vocabulary with 256-row logits chunks and every product the
-    256 x 256-tile engine can take routed there (GN_GEMM_WIDE_MIN=1): the
+    wide-tile engine can take routed there (GN_GEMM_WIDE_MIN=1): the
     lm_head forward, its input gradient (K = 65536, split) and weight
     gradient at the benchmark's V."""
     cfg, w = d12v
@@ -444,11 +469,11 @@ def _wide_launches(cfg, w, B, T, prompt_len, env, monkeypatch, seed=7):
 @pytest.mark.parametrize("parts", ["1", "3"])
 def test_latent_width_pg_step_wide_grouped_k(orc, latw, monkeypatch, parts):
     """The routed experts' weight gradients (GEMM_GROUP_K: one reduction
-    over each expert's rows) on the 256 x 256-tile engine, each expert's
+    over each expert's rows) on the wide-tile engine, each expert's
     rows cut into `parts` ranges (GN_GEMM_WIDE_PARTS; the benchmark's
     16,000-row experts take 8 by the round-filling rule) whose partials
     gemm_reduce_kernel sums into the gradient.  600 tokens give ~75 rows per
-    expert: every range ends inside a tile pair (rows past it read as
+    expert: every range ends inside a stage (rows past it read as
     zeros), and at 3 parts some experts' last range is empty.  Against the
     oracle as the other policy-gradient checks; the launch count against
     GN_GEMM_WIDE_GROUPED_K=0 shows the three weight gradients of each layer
@@ -503,6 +528,63 @@ def test_latent_width_expert_gradients_keep_their_own_range(latw, monkeypatch):
             checked += 1
             assert rel_err(pick(both)[e], pick(small)[e]) <= 1e-5, (name, e)
     assert checked >= 3, checked
+
+
+def test_latent_width_gradients_beyond_the_split(latw, monkeypatch):
+    """Gradients of about 2^112: the backward products (input and weight
+    gradients, expert-grouped rows and K) pass the bf16 parts' range and are
+    formed again on the fp32 instructions.  The step is linear in the
+    advantages, so the gradients are 2^112 times those of unit advantages, to
+    the 1e-4 bar (the two are rounded differently)."""
+    from gonano_amd.session import Session
+    cfg, w = latw
+    cfg = dataclasses.replace(cfg, balance_weight=0.0)
+    monkeypatch.setenv("GN_GEMM_WIDE_MIN", "1")
+    rng = np.random.default_rng(6)
+    inputs = rng.integers(0, cfg.vocab_size, (2, 200)).astype(np.int32)
+    targets = rng.integers(0, cfg.vocab_size, (2, 200)).astype(np.int32)
+    adv = np.array([0.7, -0.3], np.float32)
+    with Session(cfg) as s:
+        s.set_params(w)
+
+        def grads(scale):
+            s.zero_grad()
+            s.policy_gradient_step(inputs, targets, adv * np.float32(scale), 200.0)
+            return s.grads().astype(np.float64)
+
+        one, big = grads(1.0), grads(2.0 ** 112) / 2.0 ** 112
+    assert np.isfinite(big).all()
+    for name, rows, cols, off in cfg.param_table():
+        a, b = (g[off:off + rows * cols] for g in (big, one))
+        assert rel_err(a, b) <= 1e-4 or np.abs(b).max() < 1e-5 * np.abs(one).max(), name
+
+
+def test_latent_width_expert_products_on_both_engines(latw, monkeypatch):
+    """8250 tokens give 1031 rows per expert on average: the expert products
+    take the wide engine's grouped rows by size, and with GN_GEMM_WIDE=0 the 128 x
+    128 grouped tiles of gemm_kernel.  The matrices' gradients of the two agree
+    to the 1e-4 bar, the scalars (one dot product over every token and channel)
+    to the 5e-4 of _compare_grads."""
+    from gonano_amd.session import Session
+    cfg, w = latw
+    rng = np.random.default_rng(8)
+    inputs = rng.integers(0, cfg.vocab_size, (33, 250)).astype(np.int32)
+    targets = rng.integers(0, cfg.vocab_size, (33, 250)).astype(np.int32)
+    adv = rng.standard_normal(33).astype(np.float32)
+    out = []
+    for wide in ("1", "0"):
+        monkeypatch.setenv("GN_GEMM_WIDE", wide)
+        with Session(cfg) as s:
+            s.set_params(w)
+            s.set_timing(True)
+            s.zero_grad()
+            s.policy_gradient_step(inputs, targets, adv, 251.0)
+            out.append((s.grads(), s.timing()["gemm_wide_launches"]))
+    assert out[0][1] > 0 and out[1][1] == 0
+    for name, rows, cols, off in cfg.param_table():
+        a, b = (g[off:off + rows * cols] for g, _ in out)
+        tol = 1e-4 if rows * cols > 64 else 5e-4
+        assert rel_err(a, b) <= tol or np.abs(b).max() < 1e-5 * np.abs(out[1][0]).max(), name
 
 
 # ---- flash d12 width (the benchmark's flash d12 workload at 6 layers, V 4096) ---
