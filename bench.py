@@ -27,9 +27,9 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
 FP32_MFMA_PEAK_TFLOPS = 157.3
-# the wide-tile engine's fp32 products: three fp16 matrix instructions each
-# (dense fp16 peak 2.5 PFLOP/s)
-SPLIT_MFMA_PEAK_TFLOPS = 2500.0 / 3
+# the wide-tile engine's fp32 products: six bf16 matrix instructions each
+# (dense bf16 peak 2.5 PFLOP/s)
+SPLIT_MFMA_PEAK_TFLOPS = 2500.0 / 6
 METRIC = "rollout tokens/sec + RL-step ms at d12 on 1 MI355X; % of HBM/fp32-MFMA peak"
 
 WORKLOADS = {
@@ -298,8 +298,8 @@ def gemm_roofline(g: dict, config: str) -> dict:
     """The dominant kernels of the step: the train phase's fp32 products
     (recompute forward, PG backward, lm_head), timed live per launch with
     HIP events on the session stream.  Every product runs on the library's
-    own kernels: the large ones on the wide-tile engine (gemm_wide_kernel, fp16
-    matrix instructions on split operands), the rest on gemm_kernel (fp32
+    own kernels: the large ones on the wide-tile engine (gemm_wide_kernel, bf16
+    matrix instructions on fp32 operands split into three exact parts), the rest on gemm_kernel (fp32
     matrix instructions); `parts` splits the two, each against its own peak,
     and the whole is held against the rate of both parts at their peaks."""
     tf = g["flops"] / (g["ms"] / 1e3) / 1e12 if g["ms"] else 0.0
@@ -312,8 +312,8 @@ def gemm_roofline(g: dict, config: str) -> dict:
         wide["share_of_gemm_time"] = round(g["wide_ms"] / g["ms"], 4)
         own["share_of_gemm_time"] = round(1 - g["wide_ms"] / g["ms"], 4)
     return {
-        "kernel": "train-phase fp32 GEMMs (gemm_wide_kernel + gemm_kernel, all hand-written; "
-                  "recompute + PG backward + lm_head)",
+        "kernel": "train-phase fp32 GEMMs (gemm_wide_kernel, fp32 operands as three exact bf16 "
+                  "parts each, + gemm_kernel, all hand-written; recompute + PG backward + lm_head)",
         "bound": "mfma", "achieved": round(tf, 2), "peak": round(peak, 1),
         "unit": "TFLOP/s", "frac": round(tf / peak, 4),
         "traffic": gemm_traffic(config), "launches": g["n"],
