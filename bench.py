@@ -299,9 +299,10 @@ def gemm_roofline(g: dict, config: str) -> dict:
     (recompute forward, PG backward, lm_head), timed live per launch with
     HIP events on the session stream.  Every product runs on the library's
     own kernels: the large ones on the wide-tile engine (gemm_wide_kernel, bf16
-    matrix instructions on fp32 operands split into three exact parts), the rest on gemm_kernel (fp32
-    matrix instructions); `parts` splits the two, each against its own peak,
-    and the whole is held against the rate of both parts at their peaks."""
+    matrix instructions on fp32 operands split into three exact parts), the
+    rest on gemm_kernel (fp32 matrix instructions); `parts` splits the two,
+    each against its own peak, and the whole is held against the rate of both
+    parts at their peaks."""
     tf = g["flops"] / (g["ms"] / 1e3) / 1e12 if g["ms"] else 0.0
     own_flops = g["flops"] - g["wide_flops"]
     wide = _part(g["wide_ms"], g["wide_flops"], g["wide_n"], SPLIT_MFMA_PEAK_TFLOPS)

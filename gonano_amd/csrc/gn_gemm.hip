@@ -656,9 +656,9 @@ static void launch_grouped(const GemmParams& p, bool ak, bool bk, bool vec, hipS
 //
 // One 32 x BN output tile (BN = 96, 128 or 160) per workgroup of four waves
 // (2 x 2), each wave owning 16 rows x BN/2 columns: BN/32 accumulator
-// blocks, in AGPRs, by in-place inline-asm MFMAs.  A workgroup's K range is short (a few dozen 32-deep tiles), so
-// what bounds it is the latency of the first loads and of every tile's
-// loads behind the MFMAs: the tiles go through an S-stage LDS ring (S - 1
+// blocks, in AGPRs, by in-place inline-asm MFMAs.  A workgroup's K range is
+// short (a few dozen 32-deep tiles), so what bounds it is the latency of the
+// first loads and of every tile's loads behind the MFMAs: the tiles go through an S-stage LDS ring (S - 1
 // tiles in flight, one 16-24 KB stage each, up to 144 KB), enough to cover
 // ~2 us of load latency with MFMA work at one workgroup per CU.
 //
@@ -678,13 +678,14 @@ namespace slim {
 
 // One MFMA accumulating in place in an AGPR quad.  Written as inline asm so
 // that the accumulators are tied to their registers across the K loop (the
-// builtin's untied destination let register allocation rotate the 256
-// accumulators through copies inside the loop), and volatile so that the
-// memory operations placed between MFMAs keep their source order.  No
-// hazard needs wait states here: the fragments come from LDS (lgkmcnt waits
-// are inserted for the asm's operands), the accumulators are written by
-// nothing but these MFMAs, each accumulator is reused 64 MFMAs later, and
-// the epilogue reads them after a vmcnt wait and s_nops (see the kernel).
+// builtin's untied destination let register allocation rotate them through
+// copies inside the loop), and volatile so that the memory operations placed
+// between MFMAs keep their source order.  No hazard needs wait states here:
+// the fragments come from LDS (lgkmcnt waits are inserted for the asm's
+// operands), the accumulators are written by nothing but these MFMAs, an
+// accumulator is the addend of its next MFMA (NB later) in the registers it
+// was written to, which the hardware orders, and the epilogue reads them
+// after a vmcnt wait and s_nops (see the kernel).
 __device__ __forceinline__ void mfma_acc(v4f& acc, float a, float b) {
   asm volatile("v_mfma_f32_16x16x4_f32 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
 }

@@ -3,12 +3,14 @@
 //
 // Such a product reads every weight once for a few rows, so it is bound by
 // the latency of its first loads and by how much of the weight matrix is in
-// flight.  One workgroup of four waves owns 16 outputs; wave w takes a
-// quarter of the (split's) K range and requests its whole 16-row slice of
-// the weights at once (16 KV k per chunk, KV 16-byte loads per lane) beside
-// the same k of x, which stay in registers while the workgroup walks its
-// output tiles (the next tile's weights are requested before the current
-// one's sums meet).  The four partial sums meet in LDS, in wave order, in float64.
+// flight.  One workgroup of NW waves (16 where the K range and the registers
+// allow, 4 for many output tiles, whose workgroups walk several) owns 16
+// outputs; each wave takes an equal part of the (split's) K range and requests
+// its whole 16-row slice of the weights at once (16 KV k per chunk, KV 16-byte
+// loads per lane) beside the same k of x, which stay in registers while the
+// workgroup walks its output tiles (the next tile's weights are requested
+// before the current one's sums meet).  The waves' partial sums meet in LDS,
+// in wave order, in float64.
 //
 // Why: at these sizes gemm_kernel's 64 x 64 tiles ran 16-fold padding through
 // a four-stage LDS pipeline, 13.4 us per d12 projection of one decode row.

@@ -9,7 +9,7 @@ value).  The compiler inserts the required wait state for global and flat
 stores but not for buffer stores that take their offset from an SGPR, so
 kernels store through global pointers; this check keeps it that way.
 
-Inline-asm MFMA results: the wide GEMM issues its MFMAs as inline asm
+Inline-asm MFMA results: the slim-tile GEMM issues its MFMAs as inline asm
 (accumulators tied to AGPRs), which the compiler's hazard recognizer does
 not see as MFMAs, so it inserts no wait states before an instruction that
 reads or rewrites their AGPRs.  Every such access must come at least
