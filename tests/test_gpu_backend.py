@@ -305,7 +305,7 @@ def _check_split(be, a, w, bound, what):
             be.MatMul(got, a, np.ascontiguousarray(w.T), m, n, k)
         else:
             be.MatMulTransposed(got, a, w, m, n, k)
-        assert np.all(np.abs(got.astype(np.float64) - want)[fin] <= bound[fin]), (what, name)
+        assert np.all(np.abs(got[fin].astype(np.float64) - want[fin]) <= bound[fin]), (what, name)
         assert np.array_equal(got[~fin], want32[~fin], equal_nan=True), (what, name)
 
 
